@@ -13,6 +13,7 @@
 
 #include "../../include/afid.h"
 #include "afid_internal.h"
+#include "host_memory.h"
 #include "kernels.h"
 
 using namespace afid;
@@ -946,19 +947,27 @@ static int ensure_stage(afid_ctx *c, size_t bytes) {
 }
 
 // ---- host transfers
-// The device address of [p, p + bytes) if all of it is pinned host memory of one
-// allocation, else null.
-static double *pinned_address(const void *p, size_t bytes) {
-  hipPointerAttribute_t lo{}, hi{};
-  if (hipPointerGetAttributes(&lo, p) != hipSuccess ||
-      hipPointerGetAttributes(&hi, (const char *)p + bytes - 1) != hipSuccess) {
-    (void)hipGetLastError();   // an ordinary pointer: not an error of this context
-    return nullptr;
+// What the runtime knows of a host address.  An address that it does not know is
+// not an error of this context.
+static bool lookup(uintptr_t a, Allocation *o) {
+  hipPointerAttribute_t t{};
+  if (hipPointerGetAttributes(&t, (const void *)a) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
   }
-  if (lo.type != hipMemoryTypeHost || hi.type != hipMemoryTypeHost || !lo.devicePointer || !hi.devicePointer ||
-      (char *)hi.devicePointer - (char *)lo.devicePointer != (ptrdiff_t)(bytes - 1))
-    return nullptr;
-  return (double *)lo.devicePointer;
+  if (t.type == hipMemoryTypeUnregistered) return false;
+  if (t.type != hipMemoryTypeHost || !t.devicePointer || !t.hostPointer) return true;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, t.devicePointer) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  o->host = true;
+  o->device = (uintptr_t)base;
+  o->base = (uintptr_t)t.hostPointer - ((uintptr_t)t.devicePointer - (uintptr_t)base);
+  o->size = size;
+  return true;
 }
 
 // Staging buffer to the caller's memory on the context's stream, which is idle;
@@ -967,9 +976,10 @@ static double *pinned_address(const void *p, size_t bytes) {
 // the DMA into the other; the runtime's own staging does one after the
 // other (29 MB 1750 us, now 1250).  Towards the device the runtime was the
 // faster one (840 against 1220 us) and is left to it.
-static int copy_to_host(afid_ctx *c, void *host, const void *dev, size_t bytes) {
+// Memory that is not the host's own (kind other) is the runtime's to write.
+static int copy_to_host(afid_ctx *c, void *host, const void *dev, size_t bytes, HostKind kind) {
   Transfer &x = c->xf;
-  const bool staged = bytes >= 4 * XF_CHUNK && !pinned_address(host, bytes);
+  const bool staged = bytes >= 4 * XF_CHUNK && kind == HostKind::ordinary;
   if (staged && !x.pin && hipHostMalloc((void **)&x.pin, 2 * XF_CHUNK) != hipSuccess) {
     x.pin = nullptr;
     (void)hipGetLastError();
@@ -1058,7 +1068,9 @@ int afid_download(afid_ctx *c, int field, double *host, int ld1, int ld2, int j0
   // rate of the link (54.7 GB/s) and without a staging buffer: 43 us a field
   // through it at 32x64x64, now 32, 183 and 167 at 64x128x128; a large field
   // takes as long as before (33.3 ms at 384x768x768).
-  double *pinned = dense ? pinned_address(host, bytes) : nullptr;
+  uintptr_t device = 0;
+  const HostKind kind = host_kind(host, bytes, lookup, &device);
+  double *pinned = dense && kind == HostKind::pinned && device % sizeof(double) == 0 ? (double *)device : nullptr;
   if (!pinned) {
     if ((rc = ensure_stage(c, bytes))) return rc;
     if (!dense) HIPCHK(c, hipMemsetAsync(c->stage, 0, bytes, c->st));
@@ -1071,7 +1083,7 @@ int afid_download(afid_ctx *c, int field, double *host, int ld1, int ld2, int j0
   if ((rc = kerr(c, launch_scatter_out(src, pinned ? pinned : c->stage, c->g, n1, ld1, ld2, j0, i0, halo, c->st))))
     return rc;
   HIPCHK(c, hipStreamSynchronize(c->st));
-  if (!pinned && (rc = copy_to_host(c, host, c->stage, bytes))) return rc;
+  if (!pinned && (rc = copy_to_host(c, host, c->stage, bytes, kind))) return rc;
   if (field == AFID_RHS) {
     std::vector<double> plane((size_t)c->g.ncol);
     HIPCHK(c, hipMemcpy(plane.data(), c->stale, sizeof(double) * plane.size(), hipMemcpyDeviceToHost));
