@@ -804,7 +804,10 @@ int afid_create(afid_ctx **out, const afid_params *p, const afid_metrics *m) {
   for (int q = 0; q < 4; q++) TRY(alloc_field(c, &c->bp[q]));
   // The second pr array, where the cell's other allocations (spectrum, staging)
   // still fit beside it; without it the corrections are passes of their own.
-  if (second_pr(p, field_bytes(c))) {
+  // AFID_CORRECT=apart: such a cell, whatever the memory; its steps give the same bits.
+  const char *cenv = std::getenv("AFID_CORRECT");
+  const bool apart = cenv && std::strcmp(cenv, "apart") == 0;
+  if (second_pr(p, field_bytes(c)) && !apart) {
     size_t room = 0, total = 0;
     if (hipMemGetInfo(&room, &total) != hipSuccess || room < 4 * field_bytes(c) || alloc_field(c, &c->pr2) != AFID_OK)
       (void)hipGetLastError();
@@ -1291,10 +1294,7 @@ static FusedArgs update_args(afid_ctx *c, int ns, bool dev, bool corrects = fals
 // stencil passes of substeps 2 and 3 may make the corrections before them.
 static int enqueue_substep(afid_ctx *c, int ns, bool dev, bool cfl_fold = false, bool whole_step = false) {
   int rc;
-  // Host-driven steps of the mixed mode keep the passes apart: that stencil
-  // instance rounds the right-hand sides in another order, and an FP32 spectrum
-  // makes 1e-8 of a last bit.
-  const bool fuse = whole_step && c->pr2 && (dev || !c->mixed);
+  const bool fuse = whole_step && c->pr2;
   FusedArgs a = update_args(c, ns, dev, fuse && ns > 1);
   const bool apart = cfl_fold;
   if (apart) {

@@ -264,6 +264,15 @@ __device__ __forceinline__ double corr_pr(double pr, double d, double dkm, doubl
   return __builtin_fma(-be, __builtin_fma(z, dzq, y * dyq) + x, pr + d);
 }
 
+// One rounding of a b + c, and a b - c d with the second product rounded first.
+template <typename E = double>
+__device__ __forceinline__ E fma_(E a, E b, E c) {
+  if constexpr (std::is_same<E, float>::value) return __builtin_fmaf(a, b, c);
+  else return __builtin_fma(a, b, c);
+}
+template <typename E>
+__device__ __forceinline__ E pdiff(E a, E b, E c, E d) { return fma_<E>(a, b, -(c * d)); }
+
 // DEV: the substep scalars come from the device step state (a.ds) rather
 // than from the argument block; two instantiations keep each one's scalar
 // loads unconditional.
@@ -511,6 +520,10 @@ __global__ void __launch_bounds__(SY_WG)
       if (k == 0) stalep[(int64_t)ic * g.nym + jc] = vzc;   // the column solve reads it there, then writes the row
     }
     if (stv) {
+// Which products are fused is written out, here as in the correction: left to
+// the compiler, an instance may fuse another product of a sum than its siblings,
+// and a cell's result would hang on the route that its steps take.
+#pragma clang fp contract(off)
       // The explicit terms in E: FP64, or FP32 in the mixed-precision mode (their
       // inputs rounded from the FP64 fields); the right-hand sides, b' and the
       // solves stay FP64.  With E = double the expressions are the FP64 ones.
@@ -525,18 +538,17 @@ __global__ void __launch_bounds__(SY_WG)
       const E Eudzq_re = c.udzq_re, Eudyq_re = c.udyq_re, Eudzq_pe = c.udzq_pe, Eudyq_pe = c.udyq_pe;
       // ---- vx (ExplicitTermsVX.F90:55-101, ImplicitAndUpdateVX.F90:47-60)
       {
-        E hxz = (((Evzip + Evzipm) * (Evxip + Evxc)) - ((Evzc + Evzm) * (Evxc + Evxim))) * Eudz4;
-        E hxy = (((Evyjp + Evyjpm) * (Evxjp + Evxc)) - ((Evyc + Evym) * (Evxc + Evxjm))) * Eudy4;
-        E aa = Evxp + Evxc, bb = Evxc + Evxm;
-        E hxx = (aa * aa - bb * bb) * Eudx3c * (E)0.25;
-        E dzzvx = (Evxim - (E)2.0 * Evxc + Evxip) * Eudzq_re;
-        E dyyvx = (Evxjm - (E)2.0 * Evxc + Evxjp) * Eudyq_re;
-        double q = -(hxx + hxy + hxz) + dyyvx + dzzvx + Etc;
-        double dxxvx = vxp * apc + vxc * acc + vxm * amc;
-        double dxp = (prc - prm) * (c.al * udx3c);
-        double r = USE_RU ? c.ro * rxo : 0.0;
-        double rhs = (c.ga * q + r + c.alre * dxxvx - dxp) * c.dt;
-        double vin = rhs * cfv(SC_XSC) + ((cfv(SC_XDL) * vxm + vxc) + cfv(SC_XDU) * vxp);
+        const E hxz = pdiff<E>(Evzip + Evzipm, Evxip + Evxc, Evzc + Evzm, Evxc + Evxim);   // times udz4
+        const E hxy = pdiff<E>(Evyjp + Evyjpm, Evxjp + Evxc, Evyc + Evym, Evxc + Evxjm);   // times udy4
+        const E aa = Evxp + Evxc, bb = Evxc + Evxm;
+        const E hxx = pdiff<E>(aa, aa, bb, bb) * Eudx3c;                                   // times 0.25
+        const E dzzvx = Evxim - (E)2.0 * Evxc + Evxip, dyyvx = Evxjm - (E)2.0 * Evxc + Evxjp;
+        const E hx = fma_<E>(hxz, Eudz4, fma_<E>(hxx, (E)0.25, hxy * Eudy4));
+        const double q = fma_<E>(dzzvx, Eudzq_re, fma_<E>(dyyvx, Eudyq_re, -hx)) + Etc;
+        const double dxxvx = fma_(vxm, amc, fma_(vxc, acc, vxp * apc));
+        const double rq = USE_RU ? fma_(c.ro, rxo, c.ga * q) : c.ga * q + 0.0;
+        const double rhs = fma_(-(c.al * udx3c), prc - prm, fma_(c.alre, dxxvx, rq)) * c.dt;
+        const double vin = fma_(rhs, cfv(SC_XSC), fma_(cfv(SC_XDU), vxp, fma_(cfv(SC_XDL), vxm, vxc)));
         double vbd = stale0 + vxc;
         if (keep_ru) sth<H32, CM != CM_KEEP>(rux, C + sb, pad ? 0.0 : (inx ? q : 0.0));
         stf<CM == CM_STREAM>(bx, C + sb, pad ? 0.0 : (inx ? vin : vbd));
@@ -545,18 +557,17 @@ __global__ void __launch_bounds__(SY_WG)
       {
         const double vymm = k == 0 ? vyc : vym, vypp = k == nxm - 1 ? vyc : vyp;
         const E Evymm = vymm, Evypp = vypp;
-        E hyx = ((Evxp + Evxjmp) * (Evypp + Evyc) - (Evxc + Evxjm) * (Evyc + Evymm)) * Eudx3m * (E)0.25;
-        E yp = Evyjp + Evyc, ym = Evyjm + Evyc;
-        E hyy = (yp * yp - ym * ym) * Eudy4;
-        E hyz = ((Evyip + Evyc) * (Evzip + Evzjmip) - (Evyc + Evyim) * (Evzc + Evzjm)) * Eudz4;
-        E dyyvy = (Evyjp - (E)2.0 * Evyc + Evyjm) * Eudyq_re;
-        E dzzvy = (Evyip - (E)2.0 * Evyc + Evyim) * Eudzq_re;
-        double h = -(hyx + hyy + hyz) + dyyvy + dzzvy;
-        double dxxvy = vypp * aps + vyc * acs + vymm * ams;
-        double dyp = (prc - prjm) * c.udy_al;
-        double r = USE_RU ? c.ro * ryo : 0.0;
-        double rhs = (c.ga * h + r + c.alre * dxxvy - dyp) * c.dt;
-        double vin = rhs * cfv(SC_YSC) + ((cfv(SC_YDL) * vym + vyc) + cfv(SC_YDU) * vyp);
+        const E hyx = pdiff<E>(Evxp + Evxjmp, Evypp + Evyc, Evxc + Evxjm, Evyc + Evymm) * Eudx3m;   // times 0.25
+        const E yp = Evyjp + Evyc, ym = Evyjm + Evyc;
+        const E hyy = pdiff<E>(yp, yp, ym, ym);                                                     // times udy4
+        const E hyz = pdiff<E>(Evyip + Evyc, Evzip + Evzjmip, Evyc + Evyim, Evzc + Evzjm);          // times udz4
+        const E dyyvy = Evyjp - (E)2.0 * Evyc + Evyjm, dzzvy = Evyip - (E)2.0 * Evyc + Evyim;
+        const E hy = fma_<E>(hyz, Eudz4, fma_<E>(hyy, Eudy4, hyx * (E)0.25));
+        const double h = fma_<E>(dzzvy, Eudzq_re, fma_<E>(dyyvy, Eudyq_re, -hy));
+        const double dxxvy = fma_(vymm, ams, fma_(vyc, acs, vypp * aps));
+        const double rq = USE_RU ? fma_(c.ro, ryo, c.ga * h) : c.ga * h + 0.0;
+        const double rhs = fma_(-(prc - prjm), c.udy_al, fma_(c.alre, dxxvy, rq)) * c.dt;
+        const double vin = fma_(rhs, cfv(SC_YSC), fma_(cfv(SC_YDU), vyp, fma_(cfv(SC_YDL), vym, vyc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(ruy, C + sb, pad ? 0.0 : (iny ? h : 0.0));
         stf<CM == CM_STREAM>(by, C + sb, pad ? 0.0 : vin);   // row nx-1 is outside the nxm system and never read
       }
@@ -564,33 +575,32 @@ __global__ void __launch_bounds__(SY_WG)
       {
         const double vzmm = k == 0 ? vzc : vzm, vzpp = k == nxm - 1 ? vzc : vzp;
         const E Evzmm = vzmm, Evzpp = vzpp;
-        E zp = Evzip + Evzc, zm = Evzim + Evzc;
-        E hzz = (zp * zp - zm * zm) * Eudz4;
-        E hzy = ((Evyjp + Evyjpim) * (Evzjp + Evzc) - (Evyc + Evyim) * (Evzc + Evzjm)) * Eudy4;
-        E hzx = ((Evxp + Evximp) * (Evzpp + Evzc) - (Evxc + Evxim) * (Evzc + Evzmm)) * Eudx3m * (E)0.25;
-        E dzzvz = (Evzip - (E)2.0 * Evzc + Evzim) * Eudzq_re;
-        E dyyvz = (Evzjp - (E)2.0 * Evzc + Evzjm) * Eudyq_re;
-        double h = -(hzx + hzy + hzz) + dyyvz + dzzvz;
-        double dxxvz = vzpp * aps + vzc * acs + vzmm * ams;
-        double dzp = (prc - prim) * c.dz * c.al;
-        double r = USE_RU ? c.ro * rzo : 0.0;
-        double rhs = (c.ga * h + r + c.alre * dxxvz - dzp) * c.dt;
-        double vin = rhs * cfv(SC_YSC) + ((cfv(SC_YDL) * vzm + vzc) + cfv(SC_YDU) * vzp);
+        const E zp = Evzip + Evzc, zm = Evzim + Evzc;
+        const E hzz = pdiff<E>(zp, zp, zm, zm);                                                     // times udz4
+        const E hzy = pdiff<E>(Evyjp + Evyjpim, Evzjp + Evzc, Evyc + Evyim, Evzc + Evzjm);          // times udy4
+        const E hzx = pdiff<E>(Evxp + Evximp, Evzpp + Evzc, Evxc + Evxim, Evzc + Evzmm) * Eudx3m;   // times 0.25
+        const E dzzvz = Evzip - (E)2.0 * Evzc + Evzim, dyyvz = Evzjp - (E)2.0 * Evzc + Evzjm;
+        const E hz = fma_<E>(hzz, Eudz4, fma_<E>(hzx, (E)0.25, hzy * Eudy4));
+        const double h = fma_<E>(dzzvz, Eudzq_re, fma_<E>(dyyvz, Eudyq_re, -hz));
+        const double dxxvz = fma_(vzmm, ams, fma_(vzc, acs, vzpp * aps));
+        const double rq = USE_RU ? fma_(c.ro, rzo, c.ga * h) : c.ga * h + 0.0;
+        const double rhs = fma_(-((prc - prim) * c.dz), c.al, fma_(c.alre, dxxvz, rq)) * c.dt;
+        const double vin = fma_(rhs, cfv(SC_YSC), fma_(cfv(SC_YDU), vzp, fma_(cfv(SC_YDL), vzm, vzc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(ruz, C + sb, pad ? 0.0 : (iny ? h : 0.0));
         stf<CM == CM_STREAM>(bz, C + sb, pad ? 0.0 : vin);
       }
       // ---- temperature (ExplicitTermsTemp.F90:52-93, ImplicitAndUpdateTemp.F90:41-54)
       {
-        E htz = ((Evzipm + Evzip) * (Etip + Etc) - (Evzm + Evzc) * (Etc + Etim)) * Eudz4;
-        E hty = ((Evyjp + Evyjpm) * (Etjp + Etc) - (Evyc + Evym) * (Etc + Etjm)) * Eudy4;
-        E htx = ((Evxp + Evxc) * (Etp + Etc) - (Evxc + Evxm) * (Etc + Etm)) * Eudx3c * (E)0.25;
-        E dzzt = (Etip - (E)2.0 * Etc + Etim) * Eudzq_pe;
-        E dyyt = (Etjp - (E)2.0 * Etc + Etjm) * Eudyq_pe;
-        double h = -(htx + hty + htz) + dyyt + dzzt;
-        double dxxt = tp * apc + tc * acc + tm * amc;
-        double r = USE_RU ? c.ro * rto : 0.0;
-        double rhs = (c.ga * h + r + c.alpec * dxxt) * c.dt;
-        double vin = rhs * cfv(SC_TSC) + ((cfv(SC_TDL) * tm + tc) + cfv(SC_TDU) * tp);
+        const E htz = pdiff<E>(Evzipm + Evzip, Etip + Etc, Evzm + Evzc, Etc + Etim);           // times udz4
+        const E hty = pdiff<E>(Evyjp + Evyjpm, Etjp + Etc, Evyc + Evym, Etc + Etjm);           // times udy4
+        const E htx = pdiff<E>(Evxp + Evxc, Etp + Etc, Evxc + Evxm, Etc + Etm) * Eudx3c;       // times 0.25
+        const E dzzt = Etip - (E)2.0 * Etc + Etim, dyyt = Etjp - (E)2.0 * Etc + Etjm;
+        const E ht = fma_<E>(htz, Eudz4, fma_<E>(htx, (E)0.25, hty * Eudy4));
+        const double h = fma_<E>(dzzt, Eudzq_pe, fma_<E>(dyyt, Eudyq_pe, -ht));
+        const double dxxt = fma_(tm, amc, fma_(tc, acc, tp * apc));
+        const double rq = USE_RU ? fma_(c.ro, rto, c.ga * h) : c.ga * h + 0.0;
+        const double rhs = fma_(c.alpec, dxxt, rq) * c.dt;
+        const double vin = fma_(rhs, cfv(SC_TSC), fma_(cfv(SC_TDU), tp, fma_(cfv(SC_TDL), tm, tc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(rut, C + sb, pad ? 0.0 : (inx ? h : 0.0));
         stf<CM == CM_STREAM>(bt, C + sb, pad ? 0.0 : (inx ? vin : tc));   // row 1 gets the vz increment added by the solve pass
       }
