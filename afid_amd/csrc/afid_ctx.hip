@@ -61,7 +61,7 @@ struct afid_ctx {
                                // after the column solve, u* (the velocities before the correction)
   // Whole steps leave the corrections of substeps 1 and 2 to the next stencil
   // pass, which reads pr of one array and writes the corrected one to the other.
-  double *pr2 = nullptr;       // the second pr array (null: every substep corrects in a pass of its own)
+  double *pr2 = nullptr;       // the second pr array, in `share` (null: every substep corrects in a pass of its own)
   StepScalars psc{};           // scalars of the substep whose correction the next stencil pass makes
   // device step control (afid_steps): step state, factorisation inputs,
   // factor rows per substep, and the captured graph of one step
@@ -77,9 +77,6 @@ struct afid_ctx {
   std::vector<double> disste_acc, dissth_acc;
   std::vector<double> lem, lec;   // cell heights of CalcDissipationNu.F90:44-55 times dx
   int nstatsamples = 0;
-  int *d_kslab = nullptr;
-  double *slab_buf = nullptr;
-  int slab_n = 0;
   double *stale = nullptr;     // rhs(1,j,i)
   double *kc = nullptr;
   double *fac_x = nullptr;     // per-routine factors (SYS_N*FR_N*ldx), current coefficients
@@ -93,8 +90,11 @@ struct afid_ctx {
   double *nat = nullptr;       // natural-order arrays: g3rc, xc, amphk, acphk, apphk, ak1, ak2, dxc, dxm
   double *partial = nullptr;
   double *out = nullptr;       // reduction results, pinned host memory
-  double *stage = nullptr;
+  double *stage = nullptr;     // staging and slabs where `share` is not there or too small
   size_t stage_bytes = 0;
+  double *share = nullptr;     // staging, slab planes and the second pr array, one at a time (take_share)
+  size_t share_bytes = 0;
+  bool share_settled = false;  // take_share has decided
   Transfer xf;
   size_t bytes_held = 0;
   bool dev_steps_ready = false;   // device step state set and the step graph captured
@@ -489,10 +489,6 @@ FieldPtrs fields(const afid_ctx *c) {
 
 size_t field_bytes(const afid_ctx *c) { return sizeof(double) * (size_t)c->g.ncol * c->g.ldx; }
 
-// RK3 cells below 4 GiB a field, whose passes take 32-bit offsets: with 64-bit
-// ones the stencil pass has no registers left for the correction.
-bool second_pr(const afid_params *p, size_t bytes) { return p->nsst >= 3 && bytes < (1ull << 32); }
-
 int alloc_field(afid_ctx *c, double **p) {
   if (*p) return AFID_OK;
   if (hipMalloc(p, field_bytes(c)) != hipSuccess) {
@@ -678,7 +674,7 @@ int afid_destroy(afid_ctx *c) {
   for (auto &pt : c->pending) destroy(pt);
   for (int q = 0; q < AFID_NFIELDS; q++) hipFree(c->f[q]);
   for (int q = 0; q < 4; q++) hipFree(c->bp[q]);
-  hipFree(c->pr2);
+  hipFree(c->share);
   for (int q = 0; q < 3; q++) hipFree(c->fac_dev[q]);
   if (c->step_graph) hipGraphExecDestroy(c->step_graph);
   drop_prof_graph(c);
@@ -686,8 +682,6 @@ int afid_destroy(afid_ctx *c) {
   hipFree(c->mc);
   hipFree(c->stat_acc);
   hipFree(c->stat_partial);
-  hipFree(c->d_kslab);
-  hipFree(c->slab_buf);
   for (int q = 0; q < 4; q++) hipFree(c->fac_sub[q]);
   void *ps[] = {c->stale, c->kc, c->fac_x, c->S, c->piv, c->nat, c->partial, c->stage,
                 c->dpy.tw, c->dpy.rev, c->dpy.post, c->dpz.tw, c->dpz.rev, c->dpz.post,
@@ -802,15 +796,11 @@ int afid_create(afid_ctx **out, const afid_params *p, const afid_metrics *m) {
     TRY(alloc_field(c, &c->f[q]));
   c->mixed = p->precision == AFID_PREC_MIXED;
   for (int q = 0; q < 4; q++) TRY(alloc_field(c, &c->bp[q]));
-  // The second pr array, where the cell's other allocations (spectrum, staging)
-  // still fit beside it; without it the corrections are passes of their own.
-  // AFID_CORRECT=apart: such a cell, whatever the memory; its steps give the same bits.
-  const char *cenv = std::getenv("AFID_CORRECT");
-  const bool apart = cenv && std::strcmp(cenv, "apart") == 0;
-  if (second_pr(p, field_bytes(c)) && !apart) {
-    size_t room = 0, total = 0;
-    if (hipMemGetInfo(&room, &total) != hipSuccess || room < 4 * field_bytes(c) || alloc_field(c, &c->pr2) != AFID_OK)
-      (void)hipGetLastError();
+  {
+    // AFID_CORRECT=apart: steps without the second pr array, as where there is no
+    // room for it; they give the same bits.
+    const char *f = std::getenv("AFID_CORRECT");
+    c->share_settled = f && std::strcmp(f, "apart") == 0;
   }
   TRYH(hipMalloc(&c->stale, sizeof(double) * g.ncol));
   c->bytes_held += sizeof(double) * g.ncol;
@@ -937,7 +927,50 @@ int afid_get_metric(afid_ctx *c, const char *name, double *out, int n) {
   return AFID_ERR_ARG;
 }
 
-static int ensure_stage(afid_ctx *c, size_t bytes) {
+// nslab slab planes of four fields, with their levels.
+static size_t slab_bytes(const Geom &g, int nslab) { return (sizeof(int) + sizeof(double) * 4 * (size_t)g.ncol) * nslab; }
+
+// Whether whole steps of a cell use a second pr array: RK3 cells below 4 GiB a
+// field, whose passes take 32-bit offsets; with 64-bit ones the stencil pass has no
+// registers left for the correction.
+static bool second_pr(int nsst, const Geom &g) { return nsst >= 3 && sizeof(double) * (size_t)g.ncol * g.ldx < (1ull << 32); }
+
+// Bytes of the buffer for staging of transfers in plain and halo layouts, up to nine
+// slab planes and the second pr array, which are never in use together.
+static size_t share_size(int nsst, const Geom &g) {
+  const size_t staging = sizeof(double) * g.nx * (g.nym + 2) * (size_t)(g.nzm + 2);
+  return std::max({staging, slab_bytes(g, 9), second_pr(nsst, g) ? sizeof(double) * (size_t)g.ncol * g.ldx : 0});
+}
+
+// The second pr array holds a value only between the second and third stencil
+// passes of one step, so it shares its memory with the staging and the slab planes,
+// whose users wait for the stream before the host or a copy writes there: a cell
+// holds no more than staging and slabs apart took.
+// Taken at the first transfer, slab or whole step, not with the cell, so that of
+// cells created together none goes without its own arrays for another's sake,
+// and only where a 32nd of the GPU's memory is still left for the small arrays
+// that cells make later.  A cell refused once stays so: its step graph is captured.
+static void take_share(afid_ctx *c) {
+  if (c->share_settled) return;
+  c->share_settled = true;
+  if (!second_pr(c->p.nsst, c->g)) return;
+  const size_t bytes = share_size(c->p.nsst, c->g);
+  size_t room = 0, total = 0;
+  if (hipMemGetInfo(&room, &total) != hipSuccess || room < bytes + total / 32 || hipMalloc(&c->share, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    c->share = nullptr;
+    return;
+  }
+  c->share_bytes = bytes;
+  c->bytes_held += bytes;
+  c->pr2 = c->share;
+}
+
+static int ensure_stage(afid_ctx *c, size_t bytes, double **stage) {
+  take_share(c);
+  *stage = c->share;
+  if (bytes <= c->share_bytes) return AFID_OK;
+  *stage = c->stage;
   if (c->stage_bytes >= bytes) return AFID_OK;
   hipFree(c->stage);
   c->bytes_held -= c->stage_bytes;
@@ -946,6 +979,7 @@ static int ensure_stage(afid_ctx *c, size_t bytes) {
   if (hipMalloc(&c->stage, bytes) != hipSuccess) return AFID_ERR_NOMEM;
   c->bytes_held += bytes;
   c->stage_bytes = bytes;
+  *stage = c->stage;
   return AFID_OK;
 }
 
@@ -1034,13 +1068,14 @@ int afid_upload(afid_ctx *c, int field, const double *host, int ld1, int ld2, in
   if (rc) return rc;
   if (field == AFID_QCAP || field == AFID_DQ || field == AFID_HRO || field == AFID_RHS)
     if ((rc = alloc_field(c, &c->f[field]))) return rc;
-  if ((rc = ensure_stage(c, n * sizeof(double)))) return rc;
+  double *stage;
+  if ((rc = ensure_stage(c, n * sizeof(double), &stage))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->st));
-  HIPCHK(c, hipMemcpy(c->stage, host, n * sizeof(double), hipMemcpyHostToDevice));
+  HIPCHK(c, hipMemcpy(stage, host, n * sizeof(double), hipMemcpyHostToDevice));
   if (c->mixed && is_history(field)) {   // FP64 layout into b' scratch, then FP32 into the history
-    if ((rc = kerr(c, launch_gather_in(c->stage, c->bp[0], c->g, c->g.nx, ld1, ld2, j0, i0, c->st)))) return rc;
+    if ((rc = kerr(c, launch_gather_in(stage, c->bp[0], c->g, c->g.nx, ld1, ld2, j0, i0, c->st)))) return rc;
     if ((rc = kerr(c, launch_convert(c->bp[0], c->f[field], c->g.ncol * c->g.ldx, 1, c->st)))) return rc;
-  } else if ((rc = kerr(c, launch_gather_in(c->stage, c->f[field], c->g, field_rows(c, field), ld1, ld2, j0, i0,
+  } else if ((rc = kerr(c, launch_gather_in(stage, c->f[field], c->g, field_rows(c, field), ld1, ld2, j0, i0,
                                             c->st)))) {
     return rc;
   }
@@ -1074,19 +1109,20 @@ int afid_download(afid_ctx *c, int field, double *host, int ld1, int ld2, int j0
   uintptr_t device = 0;
   const HostKind kind = host_kind(host, bytes, lookup, &device);
   double *pinned = dense && kind == HostKind::pinned && device % sizeof(double) == 0 ? (double *)device : nullptr;
+  double *stage = nullptr;
   if (!pinned) {
-    if ((rc = ensure_stage(c, bytes))) return rc;
-    if (!dense) HIPCHK(c, hipMemsetAsync(c->stage, 0, bytes, c->st));
+    if ((rc = ensure_stage(c, bytes, &stage))) return rc;
+    if (!dense) HIPCHK(c, hipMemsetAsync(stage, 0, bytes, c->st));
   }
   const double *src = c->f[field];
   if (c->mixed && is_history(field)) {   // FP32 history widened into b' scratch first
     if ((rc = kerr(c, launch_convert(c->f[field], c->bp[0], c->g.ncol * c->g.ldx, 0, c->st)))) return rc;
     src = c->bp[0];
   }
-  if ((rc = kerr(c, launch_scatter_out(src, pinned ? pinned : c->stage, c->g, n1, ld1, ld2, j0, i0, halo, c->st))))
+  if ((rc = kerr(c, launch_scatter_out(src, pinned ? pinned : stage, c->g, n1, ld1, ld2, j0, i0, halo, c->st))))
     return rc;
   HIPCHK(c, hipStreamSynchronize(c->st));
-  if (!pinned && (rc = copy_to_host(c, host, c->stage, bytes, kind))) return rc;
+  if (!pinned && (rc = copy_to_host(c, host, stage, bytes, kind))) return rc;
   if (field == AFID_RHS) {
     std::vector<double> plane((size_t)c->g.ncol);
     HIPCHK(c, hipMemcpy(plane.data(), c->stale, sizeof(double) * plane.size(), hipMemcpyDeviceToHost));
@@ -1339,6 +1375,7 @@ static int refine_projection(afid_ctx *c, int ns, bool dev) {
 
 int afid_time_marcher(afid_ctx *c, double dt) {
   if (!c || dt <= 0) return AFID_ERR_ARG;
+  take_share(c);
   // every substep's factorisation is checked before the first one runs, so a
   // refused step (AFID_NUM_PIVOT) leaves the fields as they were, as the
   // device step path does
@@ -1476,6 +1513,7 @@ static int dev_steps_prepare(afid_ctx *c, int ntime0, int idtv, double dt, doubl
                              double limitcfl) {
   int rc = ensure_dev_step(c);
   if (rc) return rc;
+  take_share(c);
   DevStep h{};
   h.time = c->time; h.ntime = ntime0; h.idtv = idtv; h.dtfix = dt; h.dtmin = dtmin; h.dtmax = dtmax;
   h.limitcfl = limitcfl; h.dt = dt;
@@ -1646,7 +1684,7 @@ int afid_estimate_bytes(const afid_params *p, int64_t *bytes) {
   const int64_t L = (nx + P - 1) / P, ldx = P * L, ncol = nym * nzm;
   const int64_t ldm = ((nym / 2 + 1) + 3) / 4 * 4;
   const int64_t field = 8 * ncol * ldx, fac = 8 * (int64_t)SYS_N * FR_N * ldx;
-  int64_t b = (second_pr(p, (size_t)field) ? 15 : 14) * field;   // 10 fields, 4 b' arrays, the second pr
+  int64_t b = 14 * field;                                   // 10 fields, 4 b' arrays
   b += 8 * ncol;                                            // stale row
   int np, lm;
   xsolve_shape((int)nxm, &np, &lm);
@@ -1655,11 +1693,10 @@ int afid_estimate_bytes(const afid_params *p, int64_t *bytes) {
   b += 4 * fac + 3 * fac + 8 * 7 * nx + (int64_t)sizeof(DevStep);
   b += 20 * (nym + nzm) + 16 * nym;                         // FFT tables
   b += 8 * reduce_partial_blocks() * 16;   // reduction scratch
-  b += 8 * nx * (nym + 2) * (nzm + 2);                      // staging of uploads and downloads
   Geom gs{};
-  gs.ldx = (int)ldx;
+  gs.nx = (int)nx; gs.nym = p->nym; gs.nzm = p->nzm; gs.ldx = (int)ldx; gs.ncol = ncol;
+  b += (int64_t)share_size(p->nsst, gs);                    // staging, nine slab planes, second pr array
   b += 8 * (STATS_N * nxm + (int64_t)stats_partial_doubles(gs));  // statistics
-  b += (4 + 8 * 4 * ncol) * 9;                              // nine slab planes of four fields
   *bytes = b;
   return AFID_OK;
 }
@@ -1854,24 +1891,15 @@ int afid_get_slabs(afid_ctx *c, const int *kslab, int nslab, double *out) {
   if (!c || !kslab || !out || nslab < 1 || nslab > 64) return AFID_ERR_ARG;
   for (int m = 0; m < nslab; m++)
     if (kslab[m] < 1 || kslab[m] > c->g.nxm) return AFID_ERR_ARG;
-  if (nslab > c->slab_n) {
-    hipFree(c->d_kslab);
-    hipFree(c->slab_buf);
-    c->bytes_held -= (sizeof(int) + sizeof(double) * 4 * (size_t)c->g.ncol) * c->slab_n;
-    c->d_kslab = nullptr;
-    c->slab_buf = nullptr;
-    c->slab_n = 0;
-    HIPCHK(c, hipMalloc(&c->d_kslab, sizeof(int) * nslab));
-    HIPCHK(c, hipMalloc(&c->slab_buf, sizeof(double) * 4 * (size_t)nslab * c->g.ncol));
-    c->slab_n = nslab;
-    c->bytes_held += (sizeof(int) + sizeof(double) * 4 * (size_t)c->g.ncol) * nslab;
-  }
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  HIPCHK(c, hipMemcpy(c->d_kslab, kslab, sizeof(int) * nslab, hipMemcpyHostToDevice));
-  int rc = kerr(c, launch_slabs(fields(c), c->g, c->d_kslab, nslab, c->slab_buf, c->st));
+  double *planes;
+  int rc = ensure_stage(c, slab_bytes(c->g, nslab), &planes);
   if (rc) return rc;
+  int *levels = (int *)(planes + 4 * (size_t)nslab * c->g.ncol);
   HIPCHK(c, hipStreamSynchronize(c->st));
-  HIPCHK(c, hipMemcpy(out, c->slab_buf, sizeof(double) * 4 * (size_t)nslab * c->g.ncol, hipMemcpyDeviceToHost));
+  HIPCHK(c, hipMemcpy(levels, kslab, sizeof(int) * nslab, hipMemcpyHostToDevice));
+  if ((rc = kerr(c, launch_slabs(fields(c), c->g, levels, nslab, planes, c->st)))) return rc;
+  HIPCHK(c, hipStreamSynchronize(c->st));
+  HIPCHK(c, hipMemcpy(out, planes, sizeof(double) * 4 * (size_t)nslab * c->g.ncol, hipMemcpyDeviceToHost));
   return AFID_OK;
 }
 
@@ -1976,9 +2004,10 @@ int afid_interp_field(afid_ctx *c, int field, const double *old, int nxo, int ny
   const size_t nold = (size_t)nxo * nyom * nzom;
   const size_t b_old = nold * sizeof(double), b_crd = crd.size() * sizeof(double);
   const size_t b_lohi = lohi.size() * sizeof(int);
-  int rc = ensure_stage(c, b_old + b_crd + b_lohi);
+  double *stage;
+  int rc = ensure_stage(c, b_old + b_crd + b_lohi, &stage);
   if (rc) return rc;
-  char *st = (char *)c->stage;
+  char *st = (char *)stage;
   HIPCHK(c, hipStreamSynchronize(c->st));
   HIPCHK(c, hipMemcpy(st, old, b_old, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(st + b_old, crd.data(), b_crd, hipMemcpyHostToDevice));

@@ -281,3 +281,54 @@ def test_tuned_cell_equals_untuned():
     for nm in ("vx", "vy", "vz", "temp", "pr"):
         np.testing.assert_array_equal(c.download(nm), want[nm], err_msg=nm)
     c.close()
+
+
+# The optional second pr array of RK3 steps takes no room from other cells: a cell
+# is created without it, the estimate of the required memory leaves it out, and it
+# lies in the staging and slab buffer, so that a cell that has used all of them
+# holds no more than its estimate; 14 field arrays and staging and slabs side by
+# side are what a cell took before it had the array.
+SIZES = [(5, 4, 6), (20, 16, 10), (31, 24, 20), (32, 64, 64), (40, 48, 36), (64, 40, 36), (128, 32, 48)]
+
+
+def _params(n, nsst):
+    from afid_amd.engine import CellParams
+    return CellParams(nxm=n[0], nym=n[1], nzm=n[2], nsst=nsst, istr3=6, str3=6.0, ylen=2.0, zlen=2.0, ray=1e6, pra=0.7)
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_estimate_leaves_optional_array_out(n):
+    from afid_amd.engine import estimate_bytes
+    nx, ncol = n[0] + 1, n[1] * n[2]
+    staging, slabs = 8 * nx * (n[1] + 2) * (n[2] + 2), 9 * (4 + 32 * ncol)
+    field = 8 * 16 * ((nx + 15) // 16) * ncol
+    rk3, ab2 = estimate_bytes(_params(n, 3)), estimate_bytes(_params(n, 1))
+    assert rk3 - ab2 == max(staging, slabs, field) - max(staging, slabs)
+    assert max(staging, slabs, field) <= staging + slabs
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nsst", [1, 3])
+@pytest.mark.parametrize("n", SIZES)
+def test_held_bytes_within_estimate(n, nsst):
+    from afid_amd.engine import Cell, estimate_bytes
+    c, base = Cell(_params(n, nsst)), Cell(_params(n, 1))
+    assert c.held_bytes() == base.held_bytes()
+    c.init_linear_noise(1, 1e-3)
+    want = c.download("temp", halo=True)
+    c.upload("temp", want, halo=True)
+    c.steps_async(0, 3, 1, 1e-3)
+    assert np.isfinite(c.slabs([1, n[0]])).all()
+    c.steps_more(2)
+    c.download("vx", halo=True)          # behind the queued steps, into the memory of their second pr
+    c.steps_wait()
+    c.CalcStats()
+    c.slabs([2] * 9)
+    assert c.held_bytes() <= estimate_bytes(_params(n, nsst))
+    d = Cell(_params(n, nsst))           # the same steps alone
+    d.init_linear_noise(1, 1e-3)
+    d.steps(0, 5, 1, 1e-3)
+    for nm in ("vx", "vy", "vz", "temp", "pr"):
+        np.testing.assert_array_equal(c.download(nm), d.download(nm), err_msg=nm)
+    for x in (c, base, d):
+        x.close()
