@@ -1244,10 +1244,13 @@ static int march_planes(const Geom &g, int resident, int most) {
   }
   return best;
 }
+int stencil_planes(const Geom &g, bool corrects, int zm) {
+  return march_planes(g, corrects ? STENCIL_CORR_RESIDENT : STENCIL_RESIDENT, zm > 0 ? zm : ZM_MAX);
+}
 hipError_t launch_stencil_rhs(const FusedArgs &args, hipStream_t st) {
   FusedArgs a = args;
   const int64_t n = a.g.ncol * a.g.ldx;
-  a.zm = march_planes(a.g, a.dph ? STENCIL_CORR_RESIDENT : STENCIL_RESIDENT, a.zm > 0 ? a.zm : ZM_MAX);
+  a.zm = stencil_planes(a.g, a.dph != nullptr, a.zm);
   const int zplanes = a.zm;
   const int64_t ntile = (int64_t)((a.g.nzm + zplanes - 1) / zplanes) * ((a.g.nym + ST_GC - 1) / ST_GC) *
                         ((a.g.ldx + ST_SP - 1) / ST_SP);

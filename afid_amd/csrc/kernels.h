@@ -100,6 +100,7 @@ struct PoissonArgs {
   int spec32;            // S holds FP32 complex values and the y/z FFTs run in FP32 (mixed precision)
 };
 
+int stencil_planes(const Geom &g, bool corrects, int zm);   // z planes a block takes with the limit zm
 hipError_t launch_stencil_rhs(const FusedArgs &a, hipStream_t st);
 hipError_t launch_column_solve(const FusedArgs &a, hipStream_t st);
 hipError_t launch_solve_update(const SolveArgs &a, int which, hipStream_t st);

@@ -192,9 +192,10 @@ int afid_steps_wait(afid_ctx *ctx, double *dt_last, int *errorcode, int *steps_d
 int afid_batch_steps(afid_ctx *const *cells, int ncells, int nsteps);
 /* Autotuner for the stencil pass: times at most 8, 16, 32 and 64 z planes per
  * block (not above nzm; a small cell's blocks take fewer whatever the limit)
- * on this context and keeps the fastest for its later launches; *zm receives
- * the choice.  It
- * writes the histories and scratch while timing and clears them afterwards:
+ * on this context, in the forms that its steps launch, and keeps the fastest for
+ * its later launches, of limits that launch the same blocks the largest; *zm
+ * receives the choice.  It writes the histories and scratch while timing and
+ * clears them afterwards:
  * call it before setting the initial state.  No counterpart in the
  * reference. */
 int afid_tune(afid_ctx *ctx, int *zm);
