@@ -811,24 +811,28 @@ __device__ __forceinline__ void st_stream(double *p, double v) {
 // neighbours come through LDS, which leaves six to ten loads.  The four terms
 // (vx, vy, vz, temp) took 126, 109, 107, 128 us at 128x256x256 and take 121,
 // 80, 58, 104; 20, 16, 15, 18 and 20, 13, 13, 15 at 64x128x128.
+// GC columns to a block: sixteen, or four or eight where nym holds no more, since
+// the columns left over would be idle lanes.  The four terms together at nzm = 512,
+// nxm = 128: nym = 2 17 us one point to a thread, 39 with sixteen columns, 21 with
+// four; nym = 8 36, 40 and (eight) 27; nym = 16 67 and 42.
 // Published per plane: the term's own field, then what the other columns need of
 // the transporting ones.
 constexpr int EX_N = 5;
-template <int W, bool NT>
-__global__ void __launch_bounds__(SY_WG) k_explicit(RoutineArgs a, int zplanes) {
-  __shared__ double xv[2][EX_N][SY_WG];
+template <int W, bool NT, int GC>
+__global__ void __launch_bounds__(GC * ST_SP) k_explicit(RoutineArgs a, int zplanes) {
+  __shared__ double xv[2][EX_N][GC * ST_SP];
   const Geom g = a.g;
   const int L = g.L, ldx = g.ldx, nq = ldx / ST_SP;
-  const int ngr = (g.nym + ST_GC - 1) / ST_GC, nib = (g.nzm + zplanes - 1) / zplanes;
+  const int ngr = (g.nym + GC - 1) / GC, nib = (g.nzm + zplanes - 1) / zplanes;
   const int64_t tile = xcd_block<64>((int64_t)nib * ngr * nq);
   if (tile < 0) return;
   const int q = (int)(tile % nq);
   const int64_t rest = tile / nq;
   const int gr = (int)(rest % ngr), ib = (int)(rest / ngr);
   const int tid = (int)threadIdx.x, w = tid / ST_SP;
-  const int ncols = min(ST_GC, g.nym - gr * ST_GC);
+  const int ncols = min(GC, g.nym - gr * GC);
   const bool colok = w < ncols;
-  const int jc = colok ? gr * ST_GC + w : g.nym - 1;   // idle threads read a valid column, store nothing
+  const int jc = colok ? gr * GC + w : g.nym - 1;   // idle threads read a valid column, store nothing
   const bool jp_in = w + 1 < ncols, jm_in = w > 0;
   const int jm = wrapm(jc - 1, g.nym), jp = wrapp(jc + 1, g.nym);
   const int s = q * ST_SP + tid % ST_SP, k = k_of_pos(s, L);
@@ -880,7 +884,7 @@ __global__ void __launch_bounds__(SY_WG) k_explicit(RoutineArgs a, int zplanes) 
         zjmip = vz[col_off(jm, ip, g) + s];
       }
     }
-    double (*buf)[SY_WG] = xv[par];
+    double (*buf)[GC * ST_SP] = xv[par];
     buf[0][tid] = fc;
     if (W != 1) buf[1][tid] = yc;
     if (W == 0 || W == 3) buf[2][tid] = ym;
@@ -1325,15 +1329,18 @@ static dim3 point_grid(const Geom &g) {
 static bool streams(const Geom &g) { return cache_mode(g) == CM_STREAM; }
 hipError_t launch_explicit(const RoutineArgs &a, int which, hipStream_t st) {
   const int zplanes = march_planes(a.g, EXPLICIT_RESIDENT, ZM_MAX);
-  const int64_t ntile = (int64_t)((a.g.nzm + zplanes - 1) / zplanes) * ((a.g.nym + ST_GC - 1) / ST_GC) * (a.g.ldx / ST_SP);
+  const int gc = a.g.nym <= 4 ? 4 : (a.g.nym <= 8 ? 8 : ST_GC);
+  const int64_t ntile = (int64_t)((a.g.nzm + zplanes - 1) / zplanes) * ((a.g.nym + gc - 1) / gc) * (a.g.ldx / ST_SP);
   const dim3 grid((unsigned)(((ntile + 7) / 8) * 8));
   const bool nt = streams(a.g);
-#define GO(W, NT)                                                                            \
-  if (which == W && nt == NT) {                                                              \
-    hipLaunchKernelGGL((k_explicit<W, NT>), grid, dim3(SY_WG), 0, st, a, zplanes);           \
+#define GO(W, NT, GC)                                                                        \
+  if (which == W && nt == NT && gc == GC) {                                                  \
+    hipLaunchKernelGGL((k_explicit<W, NT, GC>), grid, dim3(GC * ST_SP), 0, st, a, zplanes);  \
     return hipGetLastError();                                                                \
   }
-  GO(0, false) GO(1, false) GO(2, false) GO(3, false) GO(0, true) GO(1, true) GO(2, true) GO(3, true)
+#define GOW(NT, GC) GO(0, NT, GC) GO(1, NT, GC) GO(2, NT, GC) GO(3, NT, GC)
+  GOW(false, ST_GC) GOW(true, ST_GC) GOW(false, 8) GOW(true, 8) GOW(false, 4) GOW(true, 4)
+#undef GOW
 #undef GO
   return hipErrorInvalidValue;
 }
