@@ -138,6 +138,8 @@ __device__ __forceinline__ double ldf(const double *base, OffT boff) {
 // and 394 us; 96x128x128 (14 MiB) 576, 536, 492; 117x135x150 (20 MiB) 826, 769,
 // 832; 96x192x192 (31.5 MiB) 1080, 1078, 1080; 128x256x256 (72 MiB) 2240, 2247,
 // 2270; 192x384x384 6.79, 6.87, 6.94 ms.
+// Steps that fold CalcMaxCFL into the last correction follow the same rule: 64x128x128
+// 494 us with that correction's inputs streamed, 469 without.
 enum CacheMode { CM_STREAM = 0, CM_HIST, CM_KEEP };
 static int cache_mode(const Geom &g) {
   const uint64_t field = (uint64_t)g.ncol * g.ldx * sizeof(double);
@@ -1359,14 +1361,12 @@ hipError_t launch_correct(const CorrectArgs &a, int which, hipStream_t st) {
                      ((a.g.ldx + ST_SP - 1) / ST_SP);
   const size_t shm = sizeof(double) * (CZ_ROWS * ST_SP + 2 * 2 * SY_WG);
   const dim3 grid((unsigned)(((nt + 7) / 8) * 8));
-  if (a.cflbits) {
-    if (which != 3 || a.ux == a.vx) return hipErrorInvalidValue;   // the fold needs u* apart from the fields
-    hipLaunchKernelGGL((k_correct<true, true>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
-  } else if (cache_mode(a.g) == CM_STREAM) {
-    hipLaunchKernelGGL((k_correct<false, true>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
-  } else {
-    hipLaunchKernelGGL((k_correct<false, false>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
-  }
+  const bool stream = cache_mode(a.g) == CM_STREAM;
+  if (a.cflbits && (which != 3 || a.ux == a.vx)) return hipErrorInvalidValue;   // the fold needs u* apart from the fields
+  if (a.cflbits && stream) hipLaunchKernelGGL((k_correct<true, true>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
+  else if (a.cflbits) hipLaunchKernelGGL((k_correct<true, false>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
+  else if (stream) hipLaunchKernelGGL((k_correct<false, true>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
+  else hipLaunchKernelGGL((k_correct<false, false>), grid, dim3(SY_WG), shm, st, a, which, zplanes);
   return hipGetLastError();
 }
 
