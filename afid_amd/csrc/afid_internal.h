@@ -71,7 +71,7 @@ __device__ __forceinline__ int64_t xcd_block(int64_t nblk) {
 // the block kc is kc[q*ldx + pos(k)].
 enum KCoef {
   KC_UDX3C = 0, KC_UDX3M, KC_AM3CK, KC_AC3CK, KC_AP3CK, KC_AM3SK, KC_AC3SK, KC_AP3SK,
-  KC_AMPHK, KC_ACPHK, KC_APPHK, KC_KMVPOS, KC_KPVPOS, KC_N
+  KC_AMPHK, KC_ACPHK, KC_APPHK, KC_N
 };
 
 // Factor rows of one wall-normal system (interleaved layout, length ldx):

@@ -22,21 +22,11 @@
 namespace afid {
 
 struct Nb {
-  int64_t C, CJM, CJP, CIM, CIP, CJMIP, CJPIM;
+  int64_t C, CJM, CIM;   // the column and its neighbours at j-1 and i-1
 };
 
 __device__ __forceinline__ Nb make_nb(int j, int i, const Geom &g) {
-  int jm = wrapm(j - 1, g.nym), jp = wrapp(j + 1, g.nym);
-  int im = wrapm(i - 1, g.nzm), ip = wrapp(i + 1, g.nzm);
-  Nb n;
-  n.C = col_off(j, i, g);
-  n.CJM = col_off(jm, i, g);
-  n.CJP = col_off(jp, i, g);
-  n.CIM = col_off(j, im, g);
-  n.CIP = col_off(j, ip, g);
-  n.CJMIP = col_off(jm, ip, g);
-  n.CJPIM = col_off(jp, im, g);
-  return n;
+  return {col_off(j, i, g), col_off(wrapm(j - 1, g.nym), i, g), col_off(j, wrapm(i - 1, g.nzm), g)};
 }
 
 // ---------------------------------------------------------------- RHS assembly
@@ -1370,7 +1360,7 @@ hipError_t launch_correct(const CorrectArgs &a, int which, hipStream_t st) {
   return hipGetLastError();
 }
 
-// LDS per block: SC_N*ST_SP + 2*SV_N*SY_WG doubles (stencil pass), SYS_N*RW_N*16*L (column
+// LDS per block: SC_NC*ST_SP + 2*SV_NC*SY_WG doubles (correcting stencil pass), SYS_N*RW_N*16*L (column
 // solve), 6*16*L (per-routine solve); L <= 80 keeps all within gfx950's 160 KiB.
 int max_supported_L() { return 80; }
 size_t column_lds_need(const Geom &g) {

@@ -250,20 +250,35 @@ __device__ __forceinline__ void ct_fft_stage(cplx_t<R> *lines, int ls, const dou
   if constexpr (ST + 1 < PL.nf) ct_fft_stage<R, N, NL, ST + 1, MR>(lines, ls, tw, sign, lane);
 }
 
+// Lines per wave: a stage has a quarter of a line's points or so as butterflies,
+// so a short line alone leaves lanes idle, while longer ones want more waves to
+// hide their loads.  Against two lines in y and one in z throughout, times in us:
+// y forward 22.2 -> 18.4 and inverse 12.1 -> 9.5 at 64x128x128, 48 -> 42 forward at
+// 96x192x192, 255 -> 237 and 127 -> 121 at 192x384x384, 506 -> 470 and 218 -> 208
+// in FP32 at 256x512x512, level at 384x768x768 (lines of 384).  z both ways
+// 24.3 -> 21.9 at 64x128x128 (two lines; four gave 22.0), 49 -> 36 at 117x135x150,
+// 73 -> 63 at 128x256x256 (four: 70), 158 -> 122 at 150x320x300, 205 -> 184 at
+// 192x384x384, 351 -> 347 in FP32 at 256x512x512.
+enum Axis { AX_Y, AX_Z };
+__host__ __device__ constexpr int wave_lines(Axis ax, int n) {
+  return ax == AX_Y ? (n <= 256 ? 4 : 2) : (n <= 64 ? 4 : (n <= 512 ? 2 : 1));
+}
+
 // The stages after the first.  R0, the plan's first radix, is 4 for all the
-// lengths the configurations use, whose stages are compiled for the length;
-// any other takes the runtime stages.
-template <typename R, int NL, int R0>
+// lengths the configurations use, whose stages are compiled for the length in
+// the kernels whose lines per wave it has; any other takes the runtime stages.
+template <typename R, Axis AX, int NL, int R0>
 __device__ __forceinline__ void fft_wave(cplx_t<R> *lines, int ls, const FFTPlan &pl, R sign, int lane) {
   if constexpr (R0 == 4) {
-    switch (pl.n) {
-#define CT_CASE(NN) \
-  case NN: ct_fft_stage<R, NN, NL, 1, 4>(lines, ls, pl.tw, sign, lane); return;
-      CT_CASE(768) CT_CASE(512) CT_CASE(384) CT_CASE(256) CT_CASE(192) CT_CASE(128) CT_CASE(96) CT_CASE(64)
-      CT_CASE(48) CT_CASE(32)
-#undef CT_CASE
-      default: break;
+#define CT_CASE(NN)                                                \
+  if constexpr (wave_lines(AX, NN) == NL)                          \
+    if (pl.n == NN) {                                              \
+      ct_fft_stage<R, NN, NL, 1, 4>(lines, ls, pl.tw, sign, lane); \
+      return;                                                      \
     }
+    CT_CASE(768) CT_CASE(512) CT_CASE(384) CT_CASE(256) CT_CASE(192) CT_CASE(128) CT_CASE(96) CT_CASE(64)
+    CT_CASE(48) CT_CASE(32)
+#undef CT_CASE
   }
   lds_fft_wave<R>(lines, ls, NL, pl, sign, lane);
 }
@@ -366,7 +381,7 @@ __global__ void __launch_bounds__(TK * 64 / NL) k_yfft_forward(PoissonArgs a) {
     }
   }
   __syncthreads();
-  fft_wave<R, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, py.c, (R)-1, threadIdx.x % 64);
+  fft_wave<R, AX_Y, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, py.c, (R)-1, threadIdx.x % 64);
   __syncthreads();
   // Post-processing: LPL lanes per real line q, wavenumbers m = lane + LPL t.
   // The padded wavenumbers m in [nymh, ldm) of each row store zeros, so that
@@ -452,7 +467,7 @@ __global__ void __launch_bounds__(TM * 64 / NL) k_zfft(PoissonArgs a, R sign) {
     }
   }
   __syncthreads();
-  fft_wave<R, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, a.pz, sign, threadIdx.x % 64);
+  fft_wave<R, AX_Z, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, a.pz, sign, threadIdx.x % 64);
   __syncthreads();
   // m < ldm: the padded wavenumbers carry zeros, so rows are written whole
   for (int nn = t; nn < N; nn += LPL) S[nn * a.ldm + q] = line[swz(nn, zsw)];
@@ -895,7 +910,7 @@ __global__ void __launch_bounds__(TK * 64 / NL) k_yfft_inverse(PoissonArgs a) {
     }
   }
   __syncthreads();
-  fft_wave<R, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, py.c, (R)1, threadIdx.x % 64);
+  fft_wave<R, AX_Y, NL, R0>(lds + (threadIdx.x / 64) * NL * ls, ls, py.c, (R)1, threadIdx.x % 64);
   __syncthreads();
   // positions k >= nxm (their lines were zero) store 0, so that every 128-byte
   // line of the column is written whole
@@ -929,17 +944,6 @@ static int y_lines(const PoissonArgs &a, bool inverse) {
   const int64_t blocks = (int64_t)(a.g.ldx / TK_MAX) * a.g.nzm;
   return fits && blocks >= (inverse ? 2048 : 0) ? TK_MAX : TK_MIN;
 }
-// Lines per wave: a stage has a quarter of a line's points or so as butterflies,
-// so a short line alone leaves lanes idle, while longer ones want more waves to
-// hide their loads.  Against two lines in y and one in z throughout, times in us:
-// y forward 22.2 -> 18.4 and inverse 12.1 -> 9.5 at 64x128x128, 48 -> 42 forward at
-// 96x192x192, 255 -> 237 and 127 -> 121 at 192x384x384, 506 -> 470 and 218 -> 208
-// in FP32 at 256x512x512, level at 384x768x768 (lines of 384).  z both ways
-// 24.3 -> 21.9 at 64x128x128 (two lines; four gave 22.0), 49 -> 36 at 117x135x150,
-// 73 -> 63 at 128x256x256 (four: 70), 158 -> 122 at 150x320x300, 205 -> 184 at
-// 192x384x384, 351 -> 347 in FP32 at 256x512x512.
-static int y_wave_lines(int n) { return n <= 256 ? 4 : 2; }
-static int z_wave_lines(int n) { return n <= 64 ? 4 : (n <= 512 ? 2 : 1); }
 // Most dynamic LDS of the transforms of one cell.
 size_t fft_lds_bytes(const RealPlan &py, const FFTPlan &pz) {
   const size_t y = std::max(sizeof(double2) * TK_MIN * line_stride(py.H, TK_MIN), (size_t)80 * 1024);
@@ -947,9 +951,10 @@ size_t fft_lds_bytes(const RealPlan &py, const FFTPlan &pz) {
 }
 
 // The y kernels by first radix and packing (an odd line has no factor 2 or 4;
-// a pair of rows alone, nym = 2, is a line of one point), the z kernel by first
-// radix.
-#define AFID_Y_LIST(X) X(4, true) X(2, true) X(3, true) X(5, true) X(1, true) X(3, false) X(5, false)
+// a pair of rows alone, nym = 2, is a line of one point and shares its wave with
+// three others), the z kernel by first radix and lines per wave.
+#define AFID_Y_LIST(X) X(4, true) X(2, true) X(3, true) X(5, true) X(3, false) X(5, false)
+#define AFID_Y_LIST4(X) AFID_Y_LIST(X) X(1, true)
 #define AFID_Z_LIST(X) X(4, 1) X(2, 1) X(3, 1) X(5, 1) X(4, 2) X(2, 2) X(3, 2) X(5, 2) X(4, 4) X(2, 4) X(3, 4) X(5, 4)
 
 // Dynamic LDS above 64 KiB must be opted into per kernel (gfx950: 160 KiB per workgroup).
@@ -959,12 +964,15 @@ static hipError_t fft_configure_lds_r(size_t bytes) {
 #define SETF(F)                                                                                                  \
   if (e == hipSuccess) e = hipFuncSetAttribute((const void *)F, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 #define SETY2(R0, HALF, TK, NL) SETF((k_yfft_forward<R, R0, HALF, TK, NL>)) SETF((k_yfft_inverse<R, R0, HALF, TK, NL>))
-#define SETY(R0, HALF) SETY2(R0, HALF, 8, 2) SETY2(R0, HALF, 16, 2) SETY2(R0, HALF, 8, 4) SETY2(R0, HALF, 16, 4)
+#define SETL2(R0, HALF) SETY2(R0, HALF, 8, 2) SETY2(R0, HALF, 16, 2)
+#define SETL4(R0, HALF) SETY2(R0, HALF, 8, 4) SETY2(R0, HALF, 16, 4)
 #define SETZ(R0, NL) SETF((k_zfft<R, R0, NL>))
-  AFID_Y_LIST(SETY)
+  AFID_Y_LIST(SETL2)
+  AFID_Y_LIST4(SETL4)
   AFID_Z_LIST(SETZ)
 #undef SETZ
-#undef SETY
+#undef SETL4
+#undef SETL2
 #undef SETY2
 #undef SETF
   return e;
@@ -997,13 +1005,14 @@ static hipError_t launch_yfft_r(const PoissonArgs &a, bool inverse, hipStream_t 
     return hipGetLastError();                                                                                 \
   }
   AFID_Y_LIST(GO)
+  if constexpr (NL == 4) GO(1, true)
 #undef GO
   return hipErrorInvalidValue;
 }
 template <typename R>
 static hipError_t launch_yfft_t(const PoissonArgs &a, bool inverse, hipStream_t st) {
   const bool wide = y_lines(a, inverse) == TK_MAX;
-  if (y_wave_lines(a.py.H) == 4)
+  if (wave_lines(AX_Y, a.py.H) == 4)
     return wide ? launch_yfft_r<R, TK_MAX, 4>(a, inverse, st) : launch_yfft_r<R, TK_MIN, 4>(a, inverse, st);
   return wide ? launch_yfft_r<R, TK_MAX, 2>(a, inverse, st) : launch_yfft_r<R, TK_MIN, 2>(a, inverse, st);
 }
@@ -1014,7 +1023,7 @@ hipError_t launch_yfft_forward(const PoissonArgs &a, hipStream_t st) { return la
 hipError_t launch_yfft_inverse(const PoissonArgs &a, hipStream_t st) { return launch_yfft(a, true, st); }
 template <typename R>
 static hipError_t launch_zfft_r(const PoissonArgs &a, int sign, dim3 grid, size_t shm, hipStream_t st) {
-  const int r0 = first_radix(a.pz), nl = z_wave_lines(a.pz.n);
+  const int r0 = first_radix(a.pz), nl = wave_lines(AX_Z, a.pz.n);
 #define GO(R0, NL)                                                                                            \
   if (r0 == R0 && nl == NL) {                                                                                 \
     hipLaunchKernelGGL((k_zfft<R, R0, NL>), grid, dim3(TM * 64 / NL), shm, st, a, (R)sign);                   \
