@@ -534,11 +534,11 @@ __global__ void __launch_bounds__(SY_WG)
         const E hxy = pdiff<E>(Evyjp + Evyjpm, Evxjp + Evxc, Evyc + Evym, Evxc + Evxjm);   // times udy4
         const E aa = Evxp + Evxc, bb = Evxc + Evxm;
         const E hxx = pdiff<E>(aa, aa, bb, bb) * Eudx3c;                                   // times 0.25
-        const E dzzvx = Evxim - (E)2.0 * Evxc + Evxip, dyyvx = Evxjm - (E)2.0 * Evxc + Evxjp;
+        const E dzzvx = fma_<E>((E)-2.0, Evxc, Evxim) + Evxip, dyyvx = fma_<E>((E)-2.0, Evxc, Evxjm) + Evxjp;
         const E hx = fma_<E>(hxz, Eudz4, fma_<E>(hxx, (E)0.25, hxy * Eudy4));
         const double q = fma_<E>(dzzvx, Eudzq_re, fma_<E>(dyyvx, Eudyq_re, -hx)) + Etc;
         const double dxxvx = fma_(vxm, amc, fma_(vxc, acc, vxp * apc));
-        const double rq = USE_RU ? fma_(c.ro, rxo, c.ga * q) : c.ga * q + 0.0;
+        const double rq = USE_RU ? fma_(c.ro, rxo, c.ga * q) : fma_(c.ga, q, 0.0);
         const double rhs = fma_(-(c.al * udx3c), prc - prm, fma_(c.alre, dxxvx, rq)) * c.dt;
         const double vin = fma_(rhs, cfv(SC_XSC), fma_(cfv(SC_XDU), vxp, fma_(cfv(SC_XDL), vxm, vxc)));
         double vbd = stale0 + vxc;
@@ -553,11 +553,11 @@ __global__ void __launch_bounds__(SY_WG)
         const E yp = Evyjp + Evyc, ym = Evyjm + Evyc;
         const E hyy = pdiff<E>(yp, yp, ym, ym);                                                     // times udy4
         const E hyz = pdiff<E>(Evyip + Evyc, Evzip + Evzjmip, Evyc + Evyim, Evzc + Evzjm);          // times udz4
-        const E dyyvy = Evyjp - (E)2.0 * Evyc + Evyjm, dzzvy = Evyip - (E)2.0 * Evyc + Evyim;
+        const E dyyvy = fma_<E>((E)-2.0, Evyc, Evyjp) + Evyjm, dzzvy = fma_<E>((E)-2.0, Evyc, Evyip) + Evyim;
         const E hy = fma_<E>(hyz, Eudz4, fma_<E>(hyy, Eudy4, hyx * (E)0.25));
         const double h = fma_<E>(dzzvy, Eudzq_re, fma_<E>(dyyvy, Eudyq_re, -hy));
         const double dxxvy = fma_(vymm, ams, fma_(vyc, acs, vypp * aps));
-        const double rq = USE_RU ? fma_(c.ro, ryo, c.ga * h) : c.ga * h + 0.0;
+        const double rq = USE_RU ? fma_(c.ro, ryo, c.ga * h) : fma_(c.ga, h, 0.0);
         const double rhs = fma_(-(prc - prjm), c.udy_al, fma_(c.alre, dxxvy, rq)) * c.dt;
         const double vin = fma_(rhs, cfv(SC_YSC), fma_(cfv(SC_YDU), vyp, fma_(cfv(SC_YDL), vym, vyc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(ruy, C + sb, pad ? 0.0 : (iny ? h : 0.0));
@@ -571,11 +571,11 @@ __global__ void __launch_bounds__(SY_WG)
         const E hzz = pdiff<E>(zp, zp, zm, zm);                                                     // times udz4
         const E hzy = pdiff<E>(Evyjp + Evyjpim, Evzjp + Evzc, Evyc + Evyim, Evzc + Evzjm);          // times udy4
         const E hzx = pdiff<E>(Evxp + Evximp, Evzpp + Evzc, Evxc + Evxim, Evzc + Evzmm) * Eudx3m;   // times 0.25
-        const E dzzvz = Evzip - (E)2.0 * Evzc + Evzim, dyyvz = Evzjp - (E)2.0 * Evzc + Evzjm;
+        const E dzzvz = fma_<E>((E)-2.0, Evzc, Evzip) + Evzim, dyyvz = fma_<E>((E)-2.0, Evzc, Evzjp) + Evzjm;
         const E hz = fma_<E>(hzz, Eudz4, fma_<E>(hzx, (E)0.25, hzy * Eudy4));
         const double h = fma_<E>(dzzvz, Eudzq_re, fma_<E>(dyyvz, Eudyq_re, -hz));
         const double dxxvz = fma_(vzmm, ams, fma_(vzc, acs, vzpp * aps));
-        const double rq = USE_RU ? fma_(c.ro, rzo, c.ga * h) : c.ga * h + 0.0;
+        const double rq = USE_RU ? fma_(c.ro, rzo, c.ga * h) : fma_(c.ga, h, 0.0);
         const double rhs = fma_(-((prc - prim) * c.dz), c.al, fma_(c.alre, dxxvz, rq)) * c.dt;
         const double vin = fma_(rhs, cfv(SC_YSC), fma_(cfv(SC_YDU), vzp, fma_(cfv(SC_YDL), vzm, vzc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(ruz, C + sb, pad ? 0.0 : (iny ? h : 0.0));
@@ -586,11 +586,11 @@ __global__ void __launch_bounds__(SY_WG)
         const E htz = pdiff<E>(Evzipm + Evzip, Etip + Etc, Evzm + Evzc, Etc + Etim);           // times udz4
         const E hty = pdiff<E>(Evyjp + Evyjpm, Etjp + Etc, Evyc + Evym, Etc + Etjm);           // times udy4
         const E htx = pdiff<E>(Evxp + Evxc, Etp + Etc, Evxc + Evxm, Etc + Etm) * Eudx3c;       // times 0.25
-        const E dzzt = Etip - (E)2.0 * Etc + Etim, dyyt = Etjp - (E)2.0 * Etc + Etjm;
+        const E dzzt = fma_<E>((E)-2.0, Etc, Etip) + Etim, dyyt = fma_<E>((E)-2.0, Etc, Etjp) + Etjm;
         const E ht = fma_<E>(htz, Eudz4, fma_<E>(htx, (E)0.25, hty * Eudy4));
         const double h = fma_<E>(dzzt, Eudzq_pe, fma_<E>(dyyt, Eudyq_pe, -ht));
         const double dxxt = fma_(tm, amc, fma_(tc, acc, tp * apc));
-        const double rq = USE_RU ? fma_(c.ro, rto, c.ga * h) : c.ga * h + 0.0;
+        const double rq = USE_RU ? fma_(c.ro, rto, c.ga * h) : fma_(c.ga, h, 0.0);
         const double rhs = fma_(c.alpec, dxxt, rq) * c.dt;
         const double vin = fma_(rhs, cfv(SC_TSC), fma_(cfv(SC_TDU), tp, fma_(cfv(SC_TDL), tm, tc)));
         if (keep_ru) sth<H32, CM != CM_KEEP>(rut, C + sb, pad ? 0.0 : (inx ? h : 0.0));
