@@ -936,7 +936,9 @@ int fft_max_len() { return 4096; }
 // inverse from 134 to 129 at 192x384x384, 642 to 525 and 269 to 219 in FP32 at
 // 256x512x512; alone on its CU it lost (the inverse 1127 against 974 us at
 // 384x768x768).  The inverse keeps eight lines while the blocks of sixteen are
-// too few to hide its stores (96x192x192, 1344 blocks: 20 against 22 us).
+// fewer than 2048: from 1150 to 3200 blocks (ten sizes, 200x96x96 to 384x128x128,
+// four of them in FP32 too) the two tiles are within 2 % of each other either way,
+// but for 48x128x512 (2048 blocks), 18.2 with eight and 17.4 with sixteen.
 constexpr int TK_MAX = 16, TK_MIN = 8;
 static int y_lines(const PoissonArgs &a, bool inverse) {
   const size_t elem = a.spec32 ? sizeof(float2) : sizeof(double2);

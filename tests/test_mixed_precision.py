@@ -112,3 +112,33 @@ def test_mixed_long_fft_lines(c):
     for nm in ("vx", "vy", "vz"):
         assert errs[nm] < 1e-4, nm
     assert errs["temp"] < 1e-7 and out[PREC_MIXED]["div"] < 1e-8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nxm,nym,nzm", [(17, 16, 5), (24, 16, 20), (33, 15, 4), (64, 40, 36), (96, 128, 160)])
+def test_mixed_host_and_device_steps(nxm, nym, nzm):
+    """Host-driven against device steps in the mixed mode, at part tiles of
+    positions and columns: each is within the mode's stated error of the FP64
+    path after 12 steps from rest (2e-5 for velocities, 1e-9 temp, 1e-6 pr), so
+    the two are within twice that of each other."""
+    from afid_amd.engine import Cell, CellParams, PREC_MIXED
+    out = []
+    for kind in ("host", "device"):
+        c = Cell(CellParams(nxm=nxm, nym=nym, nzm=nzm, istr3=6, str3=6.0, ylen=2.0, zlen=2.0, ray=1e6, pra=0.7,
+                            precision=PREC_MIXED))
+        c.init_linear_noise(9, 1e-3)
+        if kind == "host":
+            for n in range(12):
+                c.step(n, 1, 1e-3, 1e-8, 5e-3, 1.2)
+        else:
+            err, _, done = c.steps(0, 12, 1, 1e-3, 1e-8, 5e-3, 1.2)
+            assert err == 0 and done == 12
+        out.append({nm: c.download(nm) for nm in ("vx", "vy", "vz", "temp", "pr")})
+        c.close()
+    a, b = out
+    errs = {nm: rel_l2(a[nm], b[nm]) for nm in ("vx", "vy", "vz", "temp")}
+    errs["pr"] = rel_l2(demean(a["pr"][:, :, :nxm]), demean(b["pr"][:, :, :nxm]))
+    print("mixed host vs device", errs, flush=True)
+    for nm in ("vx", "vy", "vz"):
+        assert errs[nm] < 4e-5, nm
+    assert errs["temp"] < 2e-9 and errs["pr"] < 2e-6
