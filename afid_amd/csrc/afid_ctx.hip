@@ -1630,8 +1630,8 @@ int afid_batch_steps(afid_ctx *const *cells, int ncells, int nsteps) {
 }
 
 // Autotuning of the stencil pass's most z planes per block: each candidate is
-// timed with HIP events on this context's stream (one warm-up and three timed
-// launches) in the forms that a step launches: the plain one and, where whole
+// timed with HIP events on this context's stream, one warm-up and the three
+// launches of a step: the plain form, which reads the histories, and, where whole
 // steps correct in their stencil passes, twice the correcting one, whose blocks
 // are fewer at once and may take other plane counts under the same limit.  The
 // fastest is kept.  Limits that give both forms the launch shapes of a smaller one
@@ -1646,39 +1646,34 @@ int afid_tune(afid_ctx *c, int *zm_out) {
   hipEvent_t e0, e1;
   HIPCHK(c, hipEventCreate(&e0));
   HIPCHK(c, hipEventCreate(&e1));
-  FusedArgs forms[2] = {update_args(c, 2, false), update_args(c, 2, false, c->pr2 != nullptr)};
-  const int nforms = c->pr2 ? 2 : 1;
-  int best = 0, rc = AFID_OK, shape[2] = {0, 0};
+  const bool corrects = c->pr2 != nullptr;
+  FusedArgs plain = update_args(c, 2, false), second = update_args(c, 2, false, corrects);
+  plain.sc.use_ru = second.sc.use_ru = 1;
+  int best = 0, rc = AFID_OK, planes[2] = {0, 0};
   float best_ms = 0.f;
   bool was_best = false;   // the shapes timed last are the fastest so far
   for (int zm : cands) {
     if (zm > c->g.nzm && zm != cands[0]) break;   // a larger block than the grid adds nothing
-    const int planes[2] = {stencil_planes(c->g, false, zm), stencil_planes(c->g, true, zm)};
-    if (planes[0] == shape[0] && (nforms == 1 || planes[1] == shape[1])) {
+    const int np = stencil_planes(c->g, false, zm), ns = stencil_planes(c->g, corrects, zm);
+    if (np == planes[0] && ns == planes[1]) {
       if (was_best) best = zm;
       continue;
     }
-    shape[0] = planes[0];
-    shape[1] = planes[1];
-    float total = 0.f;
-    for (int q = 0; q < nforms && !rc; q++) {
-      FusedArgs &a = forms[q];
-      a.sc.use_ru = 1;
-      a.zm = zm;
-      auto launch = [&]() { return launch_stencil_rhs(a, c->st); };
-      if ((rc = kerr(c, launch()))) break;
-      if ((rc = kerr(c, hipEventRecord(e0, c->st)))) break;
-      for (int r = 0; r < 3 && !rc; r++) rc = kerr(c, launch());
-      if (rc || (rc = kerr(c, hipEventRecord(e1, c->st))) || (rc = kerr(c, hipEventSynchronize(e1)))) break;
-      float ms = 0.f;
-      if ((rc = kerr(c, hipEventElapsedTime(&ms, e0, e1)))) break;
-      total += q ? 2 * ms : ms;
-    }
-    if (rc) break;
-    was_best = best == 0 || total < best_ms;
+    planes[0] = np;
+    planes[1] = ns;
+    plain.zm = second.zm = zm;
+    if (best == 0 && (rc = kerr(c, launch_stencil_rhs(plain, c->st)))) break;
+    if ((rc = kerr(c, launch_stencil_rhs(second, c->st)))) break;
+    if ((rc = kerr(c, hipEventRecord(e0, c->st)))) break;
+    for (const FusedArgs *a : {&plain, &second, &second})
+      if (!rc) rc = kerr(c, launch_stencil_rhs(*a, c->st));
+    if (rc || (rc = kerr(c, hipEventRecord(e1, c->st))) || (rc = kerr(c, hipEventSynchronize(e1)))) break;
+    float ms = 0.f;
+    if ((rc = kerr(c, hipEventElapsedTime(&ms, e0, e1)))) break;
+    was_best = best == 0 || ms < best_ms;
     if (was_best) {
       best = zm;
-      best_ms = total;
+      best_ms = ms;
     }
   }
   hipEventDestroy(e0);
