@@ -946,7 +946,7 @@ static size_t share_size(int nsst, const Geom &g) {
 // passes of one step, so it shares its memory with the staging and the slab planes,
 // whose users wait for the stream before the host or a copy writes there: a cell
 // holds no more than staging and slabs apart took.
-// Taken at the first transfer, slab or whole step, not with the cell, so that of
+// Taken at the first transfer, slab, tuning or whole step, not with the cell, so that of
 // cells created together none goes without its own arrays for another's sake,
 // and only where a 32nd of the GPU's memory is still left for the small arrays
 // that cells make later.  A cell refused once stays so: its step graph is captured.
